@@ -163,7 +163,9 @@ typedef struct {
     int32_t n_obs;              /* obstacles (drag/lift sums are kept per obstacle) */
     const int32_t *obs_offsets_host; /* [n_obs+1] link range of each obstacle */
     int32_t ring;               /* rows of the inlet table and of the drag ring */
-    int32_t cells_per_thread;   /* 1, 2, 4 or 8 (0 = library default) */
+    int32_t cells_per_thread;   /* 1, 2, 4 or 8 (0 = library default): nodes per
+                                   work-item of the launches that advance one
+                                   iteration */
     int32_t vector_width;       /* 16-bit forms: 4 = four consecutive nodes per
                                    work-item with 8-byte accesses (taken when
                                    ny % 4 == 0 and nx*ny % (1024*cpt) == 0),
@@ -209,7 +211,9 @@ int lbm_init(lbm_fused *h, const double *g_dev, double *rho_dev, double *u_dev, 
 int lbm_step(lbm_fused *h, int64_t it, double *rho_dev, double *u_dev, void *stream);
 
 /* Iterations it0 .. it0+n-1 (it0 >= 1) without moment output, replayed from
- * a captured HIP graph. */
+ * a captured HIP graph.  A launch of the graph may advance several iterations;
+ * the last one advances one, so that iterations it0+n-2 and it0+n-1 are both
+ * in the state buffers afterwards, as with one iteration per launch. */
 int lbm_steps(lbm_fused *h, int64_t it0, int n, void *stream);
 
 /* Captures, instantiates and uploads the graph lbm_steps(h, it0, n) replays
@@ -303,10 +307,11 @@ typedef struct {
     int32_t n_cases;
     const lbm_case_desc *cases;
     int32_t storage;                /* LBM_STORE_*, common to all cases */
-    int32_t cells_per_thread;       /* tile shape, common to all cases (0 = default) */
+    int32_t cells_per_thread;       /* as lbm_fused_desc, common to all cases */
     int32_t vector_width;           /* as lbm_fused_desc */
     int32_t ring;                   /* rows of the amplitude table and drag rings */
-    int32_t grid;                   /* work-groups of the batched launch (0 = one per work item) */
+    int32_t grid;                   /* work-groups of a launch of one iteration (0 = one per
+                                       work item) */
     const double *q16_range_host;   /* LBM_STORE_Q16: as lbm_fused_desc, common to all cases */
 } lbm_batch_desc;
 

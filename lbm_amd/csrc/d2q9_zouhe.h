@@ -115,5 +115,43 @@ template <typename T> __device__ __forceinline__ void zh_corner(T *f, int which,
     f[0] = s;
 }
 
+// The same corner from the populations of the wall node beside it that its
+// wall routine reads: h = 0, 1, 2 and the three that leave through the wall
+// (4, 6, 8 at the bottom; 3, 5, 7 at the top), ux, uy that node's wall
+// velocity.  One expression for the four corners: the signs of the four cases
+// go to the velocity, where they are exact.  (The empty asm and +k: values,
+// not elements selected by address, which put the array in scratch memory.)
+template <typename T>
+__device__ __forceinline__ void zh_corner_beside(T *f, bool left, bool low, const T *h, T ux, T uy)
+{
+    T k[9];
+#pragma unroll
+    for (int q = 1; q < 9; ++q) {
+        k[q] = f[q];
+        asm("" : "+v"(k[q]));
+    }
+    const T vx = left ? ux : -ux, vy = low ? uy : -uy;
+    const T r = (h[0] + h[1] + h[2] + T(2.0) * h[3] + T(2.0) * h[4] + T(2.0) * h[5]) / (T(1.0) - vy);
+    const T kx = left ? +k[2] : +k[1], ky = low ? +k[4] : +k[3];
+    const T kl = low ? +k[6] : +k[7], kr = low ? +k[8] : +k[5];
+    const T kd = left ? +kl : +kr;
+    const T nx = kx + T(K1) * r * vx;
+    const T ny = ky + T(K1) * r * vy;
+    const T nd = kd + T(K2) * r * vx + T(K2) * r * vy;
+    const bool main = left == low;      // bottom left and top right: diagonal 5, 6
+    const T d0 = left ? +nd : +kd, d1 = left ? +kd : +nd;
+    f[1] = left ? +nx : +kx;
+    f[2] = left ? +kx : +nx;
+    f[3] = low ? +ny : +ky;
+    f[4] = low ? +ky : +ny;
+    f[5] = main ? +d0 : T(0.0);
+    f[6] = main ? +d1 : T(0.0);
+    f[7] = main ? T(0.0) : +d1;
+    f[8] = main ? T(0.0) : +d0;
+    T s = r;
+#pragma unroll
+    for (int q = 1; q < 9; ++q) s = s - f[q];
+    f[0] = s;
+}
 
 }  // namespace lbm
