@@ -424,13 +424,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W))) void k
             p, xcd_block_unit((int)blockIdx.x - eb, (int)gridDim.x - eb, 2) * 256 + threadIdx.x);
 }
 
-__global__ void k_pbb_sum_rows(const double *part, int nb, int rows, double *out)
+// Sum of a row of nb block sums, in order: a wave per row stages them in LDS,
+// work-item 0 adds (401 rows of 1024: 99 -> 17 us against one work-item per row
+// reading term by term).
+constexpr int SUM_CHUNK = 1024;
+__global__ __launch_bounds__(64) void k_pbb_sum_rows(const double *__restrict__ part, int nb,
+                                                     double *__restrict__ out)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= rows) return;
-    double s = 0.0;
-    for (int i = 0; i < nb; ++i) s += part[(size_t)r * nb + i];
-    out[r] = s;
+    __shared__ double sh[SUM_CHUNK];
+    const double *r = part + (size_t)blockIdx.x * nb;
+    double acc = 0.0;
+    for (int k0 = 0; k0 < nb; k0 += SUM_CHUNK) {
+        const int n = min(SUM_CHUNK, nb - k0);
+        for (int k = threadIdx.x; k < n; k += 64) sh[k] = r[k0 + k];
+        __syncthreads();
+        if (threadIdx.x == 0) acc = ordered_sum(sh, n, acc);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[blockIdx.x] = acc;
 }
 
 __global__ void k_zero_f64(double *p, size_t n)
@@ -606,8 +617,7 @@ extern "C" int lbm_pbb_forward(lbm_pbb *h, const void *s_dev, double u_max, doub
         fwd(h, p, st);
     }
     LBM_LAUNCH_CHECK();
-    k_pbb_sum_rows<<<(h->T + 1 + 127) / 128, 128, 0, st>>>(h->d_part, h->nblocks, h->T + 1,
-                                                          h->d_drag);
+    k_pbb_sum_rows<<<h->T + 1, 64, 0, st>>>(h->d_part, h->nblocks, h->d_drag);
     LBM_LAUNCH_CHECK();
     h->drag.assign(h->T + 1, 0.0);
     LBM_HIP_TRY(hipMemcpyAsync(h->drag.data(), h->d_drag, sizeof(double) * (h->T + 1),

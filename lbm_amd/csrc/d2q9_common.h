@@ -34,6 +34,23 @@ __host__ __device__ constexpr int xcd_block_unit(int b, int nb, int bs)
                : b;
 }
 
+// acc + v[0] + v[1] + ... + v[n - 1] in that order, by one work-item from LDS:
+// the loads of eight terms go out together, so that a term costs its addition
+// and not its latency.
+__device__ __forceinline__ double ordered_sum(const double *v, int n, double acc)
+{
+    int k = 0;
+    for (; k + 8 <= n; k += 8) {
+        double t[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t[j] = v[k + j];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc = acc + t[j];
+    }
+    for (; k < n; ++k) acc = acc + v[k];
+    return acc;
+}
+
 // Error reporting of the C ABI (per calling thread).
 int set_error(int code, const std::string &msg);
 

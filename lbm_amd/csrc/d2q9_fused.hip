@@ -665,29 +665,45 @@ __global__ __launch_bounds__(256) void k_drag_only(Params p)
     store_drag<S>(p, cell, row, f);
 }
 
-// Per-obstacle sums of the ring rows, in link plan order (nb.py:57-67).
-__global__ void k_drag_reduce(const double *__restrict__ ringbuf, int n_links, int ring,
-                              int64_t it0, int n, const int *__restrict__ obs_off, int n_obs,
-                              const int8_t *__restrict__ plan_q, double *__restrict__ out)
+// Per-obstacle sums of the ring rows, in link plan order (nb.py:57-67), one
+// wave per (iteration, obstacle): the wave forms the terms' products with the
+// components of c_q (exact: -1, 0, 1) in LDS, then work-item 0 adds the x
+// components and work-item 1 the y components one after the other.  Bound by
+// the chain of additions (~8 cycles each); one work-item per sum reading its
+// row term by term was bound by memory latency (400 iterations x 468 links:
+// 124 -> 11 us).
+constexpr int DRAG_CHUNK = 512;
+__global__ __launch_bounds__(64) void k_drag_reduce(const double *__restrict__ ringbuf, int n_links,
+                                                    int ring, int64_t it0,
+                                                    const int *__restrict__ obs_off, int n_obs,
+                                                    const int8_t *__restrict__ plan_q,
+                                                    double *__restrict__ out)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * n_obs) return;
+    __shared__ double term[2][DRAG_CHUNK];
+    const int t = blockIdx.x, lane = threadIdx.x;
     const int s = t / n_obs, o = t - s * n_obs;
     const int row = (int)((it0 + s) % ring);
     const double *r = ringbuf + (size_t)row * n_links;
-    double fx = 0.0, fy = 0.0;
-    for (int k = obs_off[o]; k < obs_off[o + 1]; ++k) {
-        const double g0 = r[k];
-        fx = fx + g0 * (double)CX[plan_q[k]];
-        fy = fy + g0 * (double)CY[plan_q[k]];
+    const int end = obs_off[o + 1];
+    double acc = 0.0;
+    for (int k0 = obs_off[o]; k0 < end; k0 += DRAG_CHUNK) {
+        const int n = min(DRAG_CHUNK, end - k0);
+        for (int k = lane; k < n; k += 64) {
+            const double g0 = r[k0 + k];
+            const int q = plan_q[k0 + k];
+            term[0][k] = g0 * (double)CX[q];
+            term[1][k] = g0 * (double)CY[q];
+        }
+        __syncthreads();
+        if (lane < 2) acc = ordered_sum(term[lane], n, acc);
+        __syncthreads();
     }
-    out[2 * (size_t)t] = fx;
-    out[2 * (size_t)t + 1] = fy;
+    if (lane < 2) out[2 * (size_t)t + lane] = acc;
 }
 
 // Density sum of one state buffer in double: FP64 sums f_q; the float forms
 // sum their stored deviations h_q in double (their populations are
-// w_q + h_q with the exact double weights w_q), and k_sum_serial adds
+// w_q + h_q with the exact double weights w_q), and k_sum_parts adds
 // N * sum_q w_q once.  Work-group partials land in part[blockIdx.x].
 template <int S>
 __global__ __launch_bounds__(256) void k_mass_partial(Params p, double *part)
@@ -719,13 +735,16 @@ __global__ __launch_bounds__(256) void k_mass_partial(Params p, double *part)
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-// out = sum of the n partials + base (the weights' share of the float forms)
-__global__ void k_sum_serial(const double *part, int n, double base, double *out)
+// out = sum of the MASS_PARTS partials in order + base (the weights' share of
+// the float forms); the partials staged in LDS (56 -> 7 us).
+constexpr int MASS_PARTS = 1024;
+__global__ __launch_bounds__(256) void k_sum_parts(const double *__restrict__ part, double base,
+                                                   double *__restrict__ out)
 {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    double s = 0.0;
-    for (int i = 0; i < n; ++i) s += part[i];
-    out[0] = s + base;
+    __shared__ double sh[MASS_PARTS];
+    for (int i = threadIdx.x; i < MASS_PARTS; i += 256) sh[i] = part[i];
+    __syncthreads();
+    if (threadIdx.x == 0) out[0] = ordered_sum(sh, MASS_PARTS, 0.0) + base;
 }
 
 __global__ void k_set_int(int *p, int v)
@@ -1720,10 +1739,9 @@ extern "C" int lbm_drag_read(lbm_fused *h, int64_t it0, int n, double *out, void
         if (int e = dmalloc(h, &h->d_drag_out, sizeof(double) * need)) return e;
         h->drag_out_cap = need;
     }
-    const int threads = n * h->n_obs;
-    k_drag_reduce<<<(threads + 127) / 128, 128, 0, S(stream)>>>(
-        h->d_drag_ring, h->n_links, h->ring, it0, n, h->d_obs_off, h->n_obs, h->d_plan_q,
-        h->d_drag_out);
+    k_drag_reduce<<<n * h->n_obs, 64, 0, S(stream)>>>(h->d_drag_ring, h->n_links, h->ring, it0,
+                                                      h->d_obs_off, h->n_obs, h->d_plan_q,
+                                                      h->d_drag_out);
     LBM_LAUNCH_CHECK();
     LBM_HIP_TRY(hipMemcpyAsync(out, h->d_drag_out, sizeof(double) * need, hipMemcpyDeviceToHost,
                                S(stream)));
@@ -1746,9 +1764,8 @@ extern "C" int lbm_drag_read_noalloc(lbm_fused *h, int64_t it0, int n, double *o
     double *stage = nullptr;
     if (int e = scratch_address(&stage)) return e;
     // k_drag_reduce writes every one of the `need` sums: nothing to clear
-    const int threads = n * h->n_obs;
-    k_drag_reduce<<<(threads + 127) / 128, 128, 0, S(stream)>>>(
-        h->d_drag_ring, h->n_links, h->ring, it0, n, h->d_obs_off, h->n_obs, h->d_plan_q, stage);
+    k_drag_reduce<<<n * h->n_obs, 64, 0, S(stream)>>>(h->d_drag_ring, h->n_links, h->ring, it0,
+                                                      h->d_obs_off, h->n_obs, h->d_plan_q, stage);
     LBM_LAUNCH_CHECK();
     LBM_HIP_TRY(hipMemcpyAsync(out, stage, sizeof(double) * need, hipMemcpyDeviceToHost,
                                S(stream)));
@@ -1796,7 +1813,7 @@ double mass_base(int storage, int N)
 extern "C" int lbm_mass(lbm_fused *h, int64_t it, double *out, void *stream)
 {
     if (!h || it < 0 || !out) return set_error(LBM_ERR_ARG, "lbm_mass: bad argument");
-    const int nb = 1024;
+    const int nb = MASS_PARTS;
     if (!h->d_part) {
         if (int e = dmalloc(h, &h->d_part, sizeof(double) * (nb + 1))) return e;
         h->n_part = nb;
@@ -1814,8 +1831,7 @@ extern "C" int lbm_mass(lbm_fused *h, int64_t it, double *out, void *stream)
     default: k_mass_partial<LBM_STORE_F16E><<<nb, 256, 0, S(stream)>>>(p, part); break;
     }
     LBM_LAUNCH_CHECK();
-    k_sum_serial<<<1, 64, 0, S(stream)>>>(h->d_part, nb, mass_base(h->storage, h->N),
-                                          h->d_part + nb);
+    k_sum_parts<<<1, 256, 0, S(stream)>>>(h->d_part, mass_base(h->storage, h->N), h->d_part + nb);
     LBM_LAUNCH_CHECK();
     LBM_HIP_TRY(hipMemcpyAsync(out, h->d_part + nb, sizeof(double), hipMemcpyDeviceToHost,
                                S(stream)));
