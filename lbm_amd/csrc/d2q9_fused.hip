@@ -40,57 +40,89 @@ int set_error(int code, const std::string &msg)
     return code;
 }
 
-// Initial and final passes, one node per work-item (grid = ceil(N/256/CPT)).
-template <int S, int MODE, int CPT>
-__global__ __launch_bounds__(256) void k_fused(Params p)
+// Iteration 0: moments and collision of g0 (null: the rest state g = w), one
+// node per work-item, grid = ceil(N / 256).
+template <int S> __global__ __launch_bounds__(256) void k_init(Params p)
+{
+    using T = typename Store<S>::T;
+    const int cell = blockIdx.x * 256 + threadIdx.x;
+    if (cell >= p.N) return;
+    T f[9];
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+        f[q] = p.g0 ? T(p.g0[(size_t)q * p.N + cell]) : weight<T>(q);
+    collide_any<S>(p, cell, f, p.rho_out != nullptr);
+}
+
+// The same from the rest state for every case of a batch, in one launch over
+// its work list (256 launches of 3.5 us before).
+template <int S>
+__global__ __launch_bounds__(256) void k_batch_init(const Params *__restrict__ cases,
+                                                    const int2 *__restrict__ work)
+{
+    using T = typename Store<S>::T;
+    const int2 item = work[blockIdx.x];
+    const Params &p = cases[2 * item.x];        // iterations of even parity write buffer 0
+    if (item.y >= p.n_main) return;             // a perimeter block
+    const int n = 1 << p.tile_shift;
+    for (int cell = item.y * n + threadIdx.x; cell < min((item.y + 1) * n, p.N); cell += 256) {
+        T f[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) f[q] = weight<T>(q);
+        collide_any<S>(p, cell, f, false);
+    }
+}
+
+// Final pass, one node per work-item: post-boundary populations of iteration
+// it and its post-collision ones, both in double.  Bound by HBM on large
+// lattices (27 planes of doubles in FP64; 8192x2048: 4.2 TB/s); the inner
+// nodes, whose pulls need no bounds, issue all their loads together, and only
+// the perimeter waits for the ring row (FP64 8192x2048 1075 -> 864 us, a
+// cavity of the 256-case FP32 batch 19.8 -> 12.6).
+template <int S> __global__ __launch_bounds__(256) void k_epilogue(Params p)
 {
     using St = Store<S>;
     using T = typename St::T;
-    const int tile = xcd_tile(blockIdx.x, gridDim.x);
-    const int base = tile * (256 * CPT) + threadIdx.x;
+    const int cell = blockIdx.x * 256 + threadIdx.x;
+    if (cell >= p.N) return;
     const int lx = p.nx - 1, ly = p.ny - 1;
-    const int row = (MODE == MODE_INIT) ? 0 : bc_row(p);
-    const bool macro = p.rho_out != nullptr;
     const auto *src = static_cast<const typename St::s_t *>(p.src);
-#pragma unroll 1
-    for (int c = 0; c < CPT; ++c) {
-        const int cell = base + c * 256;
-        if (cell >= p.N) return;
-        T f[9];
-        if (MODE == MODE_INIT) {
-            // populations of iteration 0; without an array, the rest state g = w
+    const int x = node_x(p, cell), y = cell - x * p.ny;
+    const bool interior = (unsigned)(x - 1) < (unsigned)(lx - 1) &&
+                          (unsigned)(y - 1) < (unsigned)(ly - 1);
+    T f[9];
+    double up[9];
 #pragma unroll
-            for (int q = 0; q < 9; ++q)
-                f[q] = p.g0 ? T(p.g0[(size_t)q * p.N + cell]) : weight<T>(q);
-            collide_any<S>(p, cell, f, macro);
-            continue;
+    for (int q = 0; q < 9; ++q) {
+        // the float forms' stored populations are w_q + h_q with the exact
+        // double weight w_q
+        if constexpr (S == LBM_STORE_F64) up[q] = St::ld(p, src, q, cell);
+        else up[q] = weight<double>(q) + (double)St::ldh(p, src, q, cell);
+    }
+    T r = T(0), ux = T(0), uy = T(0);
+    if (interior) {
+#pragma unroll
+        for (int q = 0; q < 9; ++q) f[q] = St::ld(p, src, q, (size_t)(cell - CX[q] * p.ny - CY[q]));
+        int lo, hi;
+        link_range(p, cell, lo, hi);
+        if (lo < hi) {
+            apply_links<S>(p, cell, lo, hi, f);
+            store_drag_range<S>(p, cell, bc_row(p), lo, hi, f);
         }
-        const int x = node_x(p, cell), y = cell - x * p.ny;
-        const bool interior = (unsigned)(x - 1) < (unsigned)(lx - 1) &&
-                              (unsigned)(y - 1) < (unsigned)(ly - 1);
-        T r = T(0), ux = T(0), uy = T(0);
+    } else {
+        const int row = bc_row(p);
         gather_bc<S>(p, x, y, cell, row, f, r, ux, uy);
         store_drag<S>(p, cell, row, f);
-        if (MODE == MODE_STEP) {
-            collide_any<S>(p, cell, f, macro);
-        } else {  // MODE_EPILOGUE
-#pragma unroll
-            for (int q = 0; q < 9; ++q) {
-                p.g_out[(size_t)q * p.N + cell] = (double)f[q];
-                // the float forms' stored populations are w_q + h_q with the
-                // exact double weight w_q
-                if constexpr (S == LBM_STORE_F64)
-                    p.gup_out[(size_t)q * p.N + cell] = St::ld(p, src, q, cell);
-                else
-                    p.gup_out[(size_t)q * p.N + cell] =
-                        weight<double>(q) + (double)St::ldh(p, src, q, cell);
-            }
-            if (!interior && p.rho_out) {
-                p.rho_out[cell] = (double)r;
-                p.u_out[cell] = (double)ux;
-                p.u_out[(size_t)p.N + cell] = (double)uy;
-            }
+        if (p.rho_out) {
+            p.rho_out[cell] = (double)r;
+            p.u_out[cell] = (double)ux;
+            p.u_out[(size_t)p.N + cell] = (double)uy;
         }
+    }
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+        p.g_out[(size_t)q * p.N + cell] = (double)f[q];
+        p.gup_out[(size_t)q * p.N + cell] = up[q];
     }
 }
 
@@ -926,13 +958,6 @@ int row_of(const lbm_fused *h, int64_t it)
     return (int)(r < 0 ? r + h->ring : r);
 }
 
-template <int S, int MODE>
-void launch_fused_s(const lbm_fused *h, const Params &p, hipStream_t s)
-{
-    const int grid = (h->N + 511) / 512;
-    k_fused<S, MODE, 2><<<grid, 256, 0, s>>>(p);
-}
-
 template <int S> void launch_step_s(const lbm_fused *h, const Params &p, hipStream_t s)
 {
     const int grid = h->n_tiles + perim_groups(h->n_perim_wg);
@@ -984,17 +1009,29 @@ void launch_step(const lbm_fused *h, const Params &p, hipStream_t s)
     }
 }
 
-template <int MODE> void launch_fused(const lbm_fused *h, const Params &p, hipStream_t s)
-{
-    switch (h->storage) {
-    case LBM_STORE_F64: launch_fused_s<LBM_STORE_F64, MODE>(h, p, s); break;
-    case LBM_STORE_F32: launch_fused_s<LBM_STORE_F32, MODE>(h, p, s); break;
-    case LBM_STORE_F16: launch_fused_s<LBM_STORE_F16, MODE>(h, p, s); break;
-    case LBM_STORE_BF16: launch_fused_s<LBM_STORE_BF16, MODE>(h, p, s); break;
-    case LBM_STORE_Q16: launch_fused_s<LBM_STORE_Q16, MODE>(h, p, s); break;
-    case LBM_STORE_F16E8: launch_fused_s<LBM_STORE_F16E8, MODE>(h, p, s); break;
-    default: launch_fused_s<LBM_STORE_F16E, MODE>(h, p, s); break;
+#define LBM_BY_FORM(storage, LAUNCH)                                             \
+    switch (storage) {                                                           \
+    case LBM_STORE_F64: LAUNCH(LBM_STORE_F64); break;                            \
+    case LBM_STORE_F32: LAUNCH(LBM_STORE_F32); break;                            \
+    case LBM_STORE_F16: LAUNCH(LBM_STORE_F16); break;                            \
+    case LBM_STORE_BF16: LAUNCH(LBM_STORE_BF16); break;                          \
+    case LBM_STORE_Q16: LAUNCH(LBM_STORE_Q16); break;                            \
+    case LBM_STORE_F16E8: LAUNCH(LBM_STORE_F16E8); break;                        \
+    default: LAUNCH(LBM_STORE_F16E); break;                                      \
     }
+
+void launch_init(const lbm_fused *h, const Params &p, hipStream_t s)
+{
+#define LAUNCH(F) k_init<F><<<(h->N + 255) / 256, 256, 0, s>>>(p)
+    LBM_BY_FORM(h->storage, LAUNCH)
+#undef LAUNCH
+}
+
+void launch_epilogue(const lbm_fused *h, const Params &p, hipStream_t s)
+{
+#define LAUNCH(F) k_epilogue<F><<<(h->N + 255) / 256, 256, 0, s>>>(p)
+    LBM_BY_FORM(h->storage, LAUNCH)
+#undef LAUNCH
 }
 
 void launch_drag_only(const lbm_fused *h, const Params &p, hipStream_t s)
@@ -1607,7 +1644,7 @@ extern "C" int lbm_init(lbm_fused *h, const double *g, double *rho, double *u, v
     p.dst = h->buf[0];
     p.rho_out = rho;
     p.u_out = u;
-    launch_fused<MODE_INIT>(h, p, S(stream));
+    launch_init(h, p, S(stream));
     LBM_LAUNCH_CHECK();
     return LBM_OK;
 }
@@ -1705,7 +1742,7 @@ extern "C" int lbm_epilogue(lbm_fused *h, int64_t it, double *g, double *gup, do
     p.k = row_of(h, it);
     p.rho_out = rho;
     p.u_out = u;
-    launch_fused<MODE_EPILOGUE>(h, p, S(stream));
+    launch_epilogue(h, p, S(stream));
     LBM_LAUNCH_CHECK();
     return LBM_OK;
 }
@@ -2086,8 +2123,10 @@ extern "C" int lbm_batch_set_amplitudes(lbm_batch *b, int64_t row0, int nrows,
 extern "C" int lbm_batch_init(lbm_batch *b, void *stream)
 {
     if (!b) return set_error(LBM_ERR_ARG, "lbm_batch_init: bad argument");
-    for (lbm_fused *h : b->cases)
-        if (int e = lbm_init(h, nullptr, nullptr, nullptr, stream)) return e;
+#define LAUNCH(F) k_batch_init<F><<<b->n_work, 256, 0, S(stream)>>>(b->d_params, b->d_work)
+    LBM_BY_FORM(b->storage, LAUNCH)
+#undef LAUNCH
+    LBM_LAUNCH_CHECK();
     return LBM_OK;
 }
 

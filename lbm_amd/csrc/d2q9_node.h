@@ -423,8 +423,6 @@ __host__ __device__ constexpr bool shifted(int S)
     return S == LBM_STORE_F16E || S == LBM_STORE_F16E8;
 }
 
-enum { MODE_INIT = 0, MODE_STEP = 1, MODE_EPILOGUE = 2, MODE_DRAG = 3 };
-
 __device__ __forceinline__ int node_x(const Params &p, int cell)
 {
     int x = (int)__umulhi((uint32_t)cell, p.magic);
@@ -808,8 +806,8 @@ __device__ __forceinline__ void collide_store_h(const Params &p, int cell, const
 
 // Work-group index -> tile index, so that each XCD (work-groups are dealt
 // round-robin over the 8 XCDs) sweeps one contiguous slab of the lattice and
-// the rows its tiles share stay in that XCD's L2 (the initial and final
-// passes; the step sweeps tiles in dispatch order, sweep_tile).
+// the rows its tiles share stay in that XCD's L2 (the multi-iteration tiles;
+// the one-iteration step sweeps its tiles in dispatch order, sweep_tile).
 // With rev set the slab is swept last tile first.
 __device__ __forceinline__ int xcd_tile(int b, int nb, int rev = 0)
 {

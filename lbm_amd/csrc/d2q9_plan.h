@@ -134,10 +134,11 @@ LBM_HD inline bool tile_perim_node(const TileRect &r, const TilePerim &P, int n,
 
 // Plans the tile of nodes [xa, xb) x [ya, yb): adds it to the plan, or its two
 // halves where a link stencil makes it larger than the shape allows.
-// near: the links (sorted as the lattice's) within 2 K + 2 nodes of the tile,
+// recip[h] = 2^32 / h.  near: the links (sorted as the lattice's) within 2 K + 2 nodes of the tile,
 // at least: a level's stencils reach two nodes beyond the next one.
 inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<const PlanLink *> &near,
-                     int cse, int xa, int xb, int ya, int yb, TilePlan &out)
+                     const std::vector<uint32_t> &recip, int cse, int xa, int xb, int ya, int yb,
+                     TilePlan &out)
 {
     static const int cx[9] = {0, 1, -1, 0, 0, 1, -1, -1, 1};
     static const int cy[9] = {0, 0, 0, 1, -1, 1, -1, 1, -1};
@@ -151,8 +152,8 @@ inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<const
     for (int l = s.K; l >= 0; --l) {
         d.r[l] = TileRect{lo_x, lo_y, hi_x - lo_x + 1, hi_y - lo_y + 1};
         const int h = d.r[l].h, hi = h - (lo_y == 0) - (hi_y == ny - 1);
-        d.mh[l] = l < s.K && h == d.r[l + 1].h ? d.mh[l + 1] : 0xffffffffu / (uint32_t)h + 1u;
-        d.mi[l] = hi == h ? d.mh[l] : hi > 1 ? 0xffffffffu / (uint32_t)hi + 1u : 0u;
+        d.mh[l] = recip[h];
+        d.mi[l] = hi > 1 ? recip[hi] : 0u;
         if (l == 0) break;
         int px = std::max(lo_x - 1, 0), qx = std::min(hi_x + 1, nx - 1);
         int py = std::max(lo_y - 1, 0), qy = std::min(hi_y + 1, ny - 1);
@@ -191,12 +192,12 @@ inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<const
         out.tiles.pop_back();
         if (xb - xa >= yb - ya) {
             const int m = (xa + xb) / 2;
-            return plan_one(nx, ny, s, near, cse, xa, m, ya, yb, out) &&
-                   plan_one(nx, ny, s, near, cse, m, xb, ya, yb, out);
+            return plan_one(nx, ny, s, near, recip, cse, xa, m, ya, yb, out) &&
+                   plan_one(nx, ny, s, near, recip, cse, m, xb, ya, yb, out);
         }
         const int m = (ya + yb) / 2;
-        return plan_one(nx, ny, s, near, cse, xa, xb, ya, m, out) &&
-               plan_one(nx, ny, s, near, cse, xa, xb, m, yb, out);
+        return plan_one(nx, ny, s, near, recip, cse, xa, xb, ya, m, out) &&
+               plan_one(nx, ny, s, near, recip, cse, xa, xb, m, yb, out);
     }
     out.max_area = std::max(out.max_area, r0.w * r0.h);
     out.max_inputs = std::max(out.max_inputs, tile_input_slots(r0, nx, ny));
@@ -302,7 +303,6 @@ inline bool plan_tiles(int nx, int ny, const TileShape &s, const std::vector<Pla
         if (links[k].x == links[k - 1].x && links[k].y == links[k - 1].y &&
             links[k].q == links[k - 1].q)
             return false;
-    out.tiles.reserve(out.tiles.size() + (size_t)s.ntx * s.nty);
     const auto tile_of = [](int v, int n, int nt) {  // tile t: [n t / nt, n (t + 1) / nt)
         v = std::min(std::max(v, 0), n - 1);
         return (int)((((int64_t)v + 1) * nt - 1) / n);
@@ -319,6 +319,8 @@ inline bool plan_tiles(int nx, int ny, const TileShape &s, const std::vector<Pla
     const int margin = 2 * s.K + 2;
     std::vector<const PlanLink *> near;
     std::vector<int> ks;
+    std::vector<uint32_t> recip(ny + 1, 0u);         // 2^32 / height
+    for (int h = 1; h <= ny; ++h) recip[h] = 0xffffffffu / (uint32_t)h + 1u;
     for (int tx = 0; tx < s.ntx; ++tx) {
         const int xa = (int)((int64_t)nx * tx / s.ntx), xb = (int)((int64_t)nx * (tx + 1) / s.ntx);
         const int ta = tile_of(xa - margin, nx, s.ntx), tb = tile_of(xb + margin, nx, s.ntx);
@@ -339,7 +341,7 @@ inline bool plan_tiles(int nx, int ny, const TileShape &s, const std::vector<Pla
             std::sort(ks.begin(), ks.end());
             near.clear();
             for (int k : ks) near.push_back(&links[k]);
-            if (!plan_one(nx, ny, s, near, cse, xa, xb, ya, yb, out)) return false;
+            if (!plan_one(nx, ny, s, near, recip, cse, xa, xb, ya, yb, out)) return false;
         }
     }
     return true;
@@ -368,6 +370,7 @@ inline const TileKind *plan_cases(const std::vector<PlanCase> &cases, bool f64, 
     for (const PlanCase &c : cases) total += (int64_t)c.nx * c.ny;
     for (int i = 0; i < n; ++i) {
         const TileKind &k = kinds[i];
+        if (!k.groups && (total > (int64_t)n_cu * k.area || (int)cases.size() > n_cu)) continue;
         // square tiles of the largest region, where there may be any number
         int side = 2;
         while ((side + 1 + 2 * k.K) * (side + 1 + 2 * k.K) <= k.area) ++side;
