@@ -56,6 +56,7 @@ struct TileShape {
     int K;                           // iterations per launch (odd: the state buffers alternate)
     int ntx, nty;                    // tiles along x and y
     int cap, nt;                     // nodes of r[0] and work-items, at most
+    bool adjoint = false;            // levels compute r[l - 1] and write into r[l]
 };
 
 struct TilePlan {
@@ -169,6 +170,11 @@ inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<const
             py = std::min(py, fy);
             qy = std::max(qy, fy);
         }
+        // a wall node beside a corner carries the corner's adjoint
+        if (s.adjoint && (py == 0 || qy == ny - 1)) {
+            if (px == 1) px = 0;
+            if (qx == nx - 2) qx = nx - 1;
+        }
         // a corner takes the density of the wall node beside it
         if (lo_y == 0 || hi_y == ny - 1) {
             if (lo_x == 0) qx = std::max(qx, std::min(2, nx - 1));
@@ -181,7 +187,7 @@ inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<const
         hi_y = qy;
     }
     const TileRect &r0 = d.r[0], &r1 = d.r[1];
-    const TilePerim P = tile_perim(r1, nx, ny);
+    const TilePerim P = tile_perim(s.adjoint ? r0 : r1, nx, ny);
     bool fits = (int64_t)r0.w * r0.h <= s.cap && P.slots <= s.nt && P.slots + P.inner <= s.cap;
     const auto inside = [&](const PlanLink &L) {
         return L.x >= r1.x && L.x < r1.x + r1.w && L.y >= r1.y && L.y < r1.y + r1.h;
@@ -270,7 +276,7 @@ struct TileKind {
 //         400^2 K5 1024x2 3.47, K5 512x2 3.92 (9.0);
 //         8192x2048 K3 512x2 237, K5 512x2 248, K5 1024x2 284, K3 512x1 307 (434)
 //   FP32  100^2 K7 512x1 1.26 (9.0); 200^2 K7 1024x2 1.45, 512x2 1.56 (8.9);
-//         512^2 K7 1024x4 2.68, K5 1024x2 2.69 (8.8); 700^2 K7 1024x4 4.03 (12.7);
+//         1073x240 (links) K5 1024x2 3.30, K7 1024x4 3.59; 700^2 K7 1024x4 4.03 (12.7);
 //         8192x2048 K5 512x4 101, K7 512x4 106, K5 512x2 114, K3 512x4 116,
 //         K5 1024x4 123 (211)
 inline const TileKind *tile_kinds(bool f64, int &n)
@@ -283,9 +289,35 @@ inline const TileKind *tile_kinds(bool f64, int &n)
     static const TileKind f[] = {{0, 7, 512, 512, 512, 0},
                                  {1, 7, 1024, 512, 640, 0},
                                  {2, 7, 2048, 1024, 2048, 0},
+                                 {2, 5, 2048, 1024, 2048, 0},
                                  {4, 7, 4096, 1024, 4096, 0},
                                  {3, 5, 2048, 512, 2048, 1}};
-    n = 5;
+    n = f64 ? 5 : 6;
+    return f64 ? d : f;
+}
+
+// The same for the launches of the channel adjoint (cfg: nodes per work-item,
+// the smallest first).  A node's adjoint takes four times the arithmetic of a
+// collision: two waves per SIMD in double (up to 256 registers each), four in
+// float; regions shrink less per CU, so K 5 rather than 7.  us per iteration,
+// recomputation included (one iteration per launch in brackets):
+//   FP64  240x64 K7 512x1 6.3, K5 6.4; 384x128 K5 512x2 7.1, K3 512x1 7.4;
+//         1024x256 K5 512x4 15.4, K3 512x3 16.0 (33);
+//         2048x512 K3 512x4 69, K5 512x4 73, K3 512x3 73
+//   FP32  240x64 K7 1024x1 5.3; 384x128 K7 1024x1 5.7, K4 5.8;
+//         768x160 K5 1024x1 7.2, K3 7.4; 1024x256 K5 1024x2 10.0, K3 10.8,
+//         K3 512x3 11.8 (27); 2048x512 K5 512x3 36.9, K3 1024x2 37.7
+inline const TileKind *adjoint_kinds(bool f64, int &n)
+{
+    static const TileKind d[] = {{0, 7, 512, 512, 512, 0},
+                                 {1, 5, 1024, 512, 1024, 0},
+                                 {2, 5, 2048, 512, 2048, 0},
+                                 {2, 3, 2048, 512, 2048, 1}};
+    static const TileKind f[] = {{0, 7, 1024, 1024, 800, 0},
+                                 {0, 5, 1024, 1024, 1024, 0},
+                                 {1, 5, 2048, 1024, 2048, 0},
+                                 {2, 5, 1536, 512, 1536, 1}};
+    n = 4;
     return f64 ? d : f;
 }
 
@@ -360,12 +392,11 @@ struct PlanCase {
 };
 
 // The plan of a set of lattices that share one launch on a GPU of n_cu CUs
-// with lds_max bytes of LDS per work-group; null when they have none.
-inline const TileKind *plan_cases(const std::vector<PlanCase> &cases, bool f64, int n_cu,
-                                  size_t lds_max, TilePlan &out)
+// with lds_max bytes of LDS per work-group, in the first of the n shapes that
+// fits; null when they have none.
+inline const TileKind *plan_cases(const std::vector<PlanCase> &cases, const TileKind *kinds, int n,
+                                  bool adjoint, bool f64, int n_cu, size_t lds_max, TilePlan &out)
 {
-    int n = 0;
-    const TileKind *kinds = tile_kinds(f64, n);
     int64_t total = 0;
     for (const PlanCase &c : cases) total += (int64_t)c.nx * c.ny;
     for (int i = 0; i < n; ++i) {
@@ -381,7 +412,7 @@ inline const TileKind *plan_cases(const std::vector<PlanCase> &cases, bool f64, 
             out = TilePlan();
             for (size_t c = 0; ok && c < cases.size(); ++c) {
                 const int nx = cases[c].nx, ny = cases[c].ny;
-                TileShape s{k.K, 0, 0, k.cap, k.nt};
+                TileShape s{k.K, 0, 0, k.cap, k.nt, adjoint};
                 if (k.groups) {
                     s.ntx = std::max(1, std::min((nx + side - 1) / side, nx / 2));
                     s.nty = std::max(1, std::min((ny + side - 1) / side, ny / 2));
@@ -399,6 +430,14 @@ inline const TileKind *plan_cases(const std::vector<PlanCase> &cases, bool f64, 
     }
     out = TilePlan();
     return nullptr;
+}
+
+inline const TileKind *plan_cases(const std::vector<PlanCase> &cases, bool f64, int n_cu,
+                                  size_t lds_max, TilePlan &out)
+{
+    int n = 0;
+    const TileKind *kinds = tile_kinds(f64, n);
+    return plan_cases(cases, kinds, n, false, f64, n_cu, lds_max, out);
 }
 
 }  // namespace lbm

@@ -115,8 +115,73 @@ static void check(int nx, int ny, int K, int cap, int nt, const std::vector<Plan
     for (int c : slots) REQUIRE(c == 1);
 }
 
+// Adjoint plans: a node's entry at a level comes from its neighbours at the
+// level before, the corner's from the wall node beside it.
+static void check_adjoint(int nx, int ny, int K, int cap, int nt, const TilePlan &plan)
+{
+    const std::vector<PlanLink> links;
+    std::vector<int> owner((size_t)nx * ny, 0);
+    for (const TileDesc &d : plan.tiles) {
+        const TileRect &o = d.r[K], &r0 = d.r[0];
+        for (int x = o.x; x < o.x + o.w; ++x)
+            for (int y = o.y; y < o.y + o.h; ++y) ++owner[(size_t)x * ny + y];
+        REQUIRE(r0.w * r0.h <= cap && r0.x >= 0 && r0.y >= 0 && r0.x + r0.w <= nx &&
+                r0.y + r0.h <= ny);
+        for (int l = K; l >= 1; --l) {
+            const TileRect &r = d.r[l], &q = d.r[l - 1];
+            for (int x = r.x; x < r.x + r.w; ++x)
+                for (int y = r.y; y < r.y + r.h; ++y)
+                    for (int k = 0; k < 9; ++k) {
+                        const int tx = x + CX[k], ty = y + CY[k];
+                        if (tx >= 0 && tx < nx && ty >= 0 && ty < ny) REQUIRE(in(q, tx, ty));
+                    }
+            for (int y : {0, ny - 1}) {
+                if (in(q, 1, y)) REQUIRE(in(q, 0, y));
+                if (in(q, nx - 2, y)) REQUIRE(in(q, nx - 1, y));
+            }
+        }
+        // launches of fewer levels start at r[1], r[2], ..
+        for (int l = 0; l < K; ++l) {
+            const TileRect &r = d.r[l];
+            const TilePerim P = tile_perim(r, nx, ny);
+            REQUIRE(P.slots <= nt && P.slots + P.inner <= cap);
+            const int hi = r.h - (r.y == 0) - (r.y + r.h == ny);
+            if (hi > 1)
+                for (int n : {0, hi - 1, hi, P.inner - 1})
+                    if (n >= 0) REQUIRE((int)(((uint64_t)n * d.mi[l]) >> 32) == n / hi);
+        }
+    }
+    for (int c : owner) REQUIRE(c == 1);
+}
+
+static void adjoint_plans()
+{
+    const int sizes[][2] = {{4, 4},     {4, 5},     {5, 9},    {33, 7},   {7, 900},   {64, 32},
+                            {150, 130}, {240, 230}, {500, 260}, {760, 440}, {1024, 256}, {4, 20000}};
+    const std::vector<PlanLink> links;
+    for (auto &sz : sizes)
+        for (int f64 = 0; f64 < 2; ++f64) {
+            const int nx = sz[0], ny = sz[1];
+            int n = 0, K = 0;
+            const TileKind *kinds = adjoint_kinds(f64, n);
+            for (int i = 0; i < n; ++i) {            // each shape by itself, then the rule
+                TilePlan plan;
+                const TileKind *k = plan_cases({{nx, ny, &links}}, kinds + i, 1, true, f64, 256,
+                                               162816, plan);
+                K = kinds[i].K;
+                REQUIRE(k || !kinds[i].groups);
+                if (k) check_adjoint(nx, ny, K, k->cap, k->nt, plan);
+            }
+            TilePlan plan;
+            const TileKind *k = plan_cases({{nx, ny, &links}}, kinds, n, true, f64, 256, 162816, plan);
+            REQUIRE(k);
+            check_adjoint(nx, ny, k->K, k->cap, k->nt, plan);
+        }
+}
+
 int main()
 {
+    adjoint_plans();
     std::mt19937 rng(7);
     const int sizes[][2] = {{4, 4},    {5, 4},    {4, 9},    {13, 200}, {64, 64},  {97, 33},
                             {100, 100}, {151, 149}, {256, 40}, {301, 299}, {541, 101}, {700, 650}};
