@@ -95,14 +95,44 @@ __host__ __device__ constexpr bool is16(int S)
            S == LBM_STORE_Q16 || S == LBM_STORE_F16E8;
 }
 
-// Float -> half conversions take their operand through an empty asm, so the
+// Float -> half conversions are written as the instruction itself, so the
 // compiler cannot fold the preceding multiply-add into a mixed-precision FMA
 // that rounds to half once (v_fma_mixlo_f16): every kernel then rounds twice,
-// to float and to half, and all kernel shapes store identical values.
+// to float and to half, and all kernel shapes store identical values.  (An
+// empty asm on the operand did the same with a register move a value.)
 __device__ __forceinline__ _Float16 to_half(float v)
 {
-    asm("" : "+v"(v));
-    return (_Float16)v;
+    uint32_t h;
+    asm("v_cvt_f16_f32 %0, %1" : "=v"(h) : "v"(v));
+    return __builtin_bit_cast(_Float16, (uint16_t)h);
+}
+// two of them in one instruction, a in the low half (each rounds as to_half)
+__device__ __forceinline__ uint32_t to_half2(float a, float b)
+{
+    uint32_t h;
+    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(h) : "v"(a), "v"(b));
+    return h;
+}
+// the low half of w (as an instruction: a conversion the compiler knows moves
+// up to the load it waits for)
+__device__ __forceinline__ float from_half(uint32_t w)
+{
+    float r;
+    asm("v_cvt_f32_f16 %0, %1" : "=v"(r) : "v"(w));
+    return r;
+}
+// e + the low / high half of w: one exact product by 1, one rounding
+__device__ __forceinline__ float add_lo(float e, uint32_t w)
+{
+    float r;
+    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(e));
+    return r;
+}
+__device__ __forceinline__ float add_hi(float e, uint32_t w)
+{
+    float r;
+    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(w), "v"(e));
+    return r;
 }
 
 // F16E: offset (in halves) of the velocity plane, 256-byte aligned
@@ -124,6 +154,14 @@ __device__ __forceinline__ void st_off(void *base, uint32_t off, E v)
     using gchar = __attribute__((address_space(1))) char;
     using gE = __attribute__((address_space(1))) E;
     *(gE *)((gchar *)base + off) = v;
+}
+// ld_off of a base that has been through sbase (a plain load of it is a flat one)
+template <class E>
+__device__ __forceinline__ E ld_base(const void *base, uint32_t off)
+{
+    using gchar = __attribute__((address_space(1))) const char;
+    using gE = __attribute__((address_space(1))) const E;
+    return *(gE *)((gchar *)base + off);
 }
 // A uniform pointer through readfirstlane: the compiler keeps each plane's
 // base in scalar registers instead of deriving one plane's address from the
@@ -376,6 +414,18 @@ __device__ __forceinline__ float e8_shift(int q, float a, float b)
     const float cu = e8_cu(q, a, b), pv = e8_pv(q, a, b);
     const float t = __builtin_fmaf(e8_k1(q), cu, e8_k2(q));
     return __builtin_fmaf(cu, t, (pv * -e8_k3(q)) * pv);
+}
+// the nine of a node: an opposite pair shares the term in pv and, up to its
+// sign, cu (the values of e8_shift)
+__device__ __forceinline__ void e8_shifts(float a, float b, float *e)
+{
+    e[0] = e8_shift(0, a, b);
+#pragma unroll
+    for (int q = 1; q < 9; q += 2) {
+        const float cu = e8_cu(q, a, b), pv = e8_pv(q, a, b), P = (pv * -e8_k3(q)) * pv;
+        e[q] = __builtin_fmaf(cu, __builtin_fmaf(cu, e8_k1(q), e8_k2(q)), P);
+        e[q + 1] = __builtin_fmaf(-cu, __builtin_fmaf(cu, -e8_k1(q), e8_k2(q)), P);
+    }
 }
 __device__ __forceinline__ float e8_dec(int q, float a, float b, float r)
 {

@@ -36,18 +36,65 @@
 namespace lbm {
 namespace {
 
-// A node's value as the pulls return it (f in FP64, h = f - w in the float
-// forms) from the planes of one state buffer.
+// A copy the compiler knows nothing about: what is derived from it inside a
+// rarely taken branch of the iteration loop is not computed ahead of the loop
+// by every work-item (in registers every wave then pays for).
+__device__ __forceinline__ int opaque(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// A node as stored, and decoded to the values the pulls return (f in FP64,
+// h = f - w in the float forms).
+template <int S> struct Raw {
+    typename Store<S>::s_t q[9];
+    uint32_t v;                                 // velocity word (shifted forms)
+};
+template <int S> __device__ __forceinline__ void tile_load(const Params &p, int cell, Raw<S> &r)
+{
+    using s_t = typename Store<S>::s_t;
+    const s_t *src = static_cast<const s_t *>(p.src);
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+        r.q[q] = ld_base<s_t>(sbase(src + (size_t)q * p.N), (uint32_t)cell * (uint32_t)sizeof(s_t));
+    if constexpr (shifted(S)) {
+        using w_t = typename Vel<S>::w_t;
+        r.v = ld_base<w_t>(sbase(Store<S>::vel(src, p.N)), (uint32_t)cell * (uint32_t)sizeof(w_t));
+    }
+}
 template <int S>
-__device__ __forceinline__ typename Store<S>::T tile_load(const Params &p, int q, int cell)
+__device__ __forceinline__ void tile_decode(const Params &p, const Raw<S> &r, typename Store<S>::T *v)
 {
     using St = Store<S>;
-    using s_t = typename St::s_t;
-    const s_t *src = static_cast<const s_t *>(p.src);
-    const s_t raw = ld_off<s_t>(src + (size_t)q * p.N, (uint32_t)cell * (uint32_t)sizeof(s_t));
-    if constexpr (S == LBM_STORE_F64 || S == LBM_STORE_F32) return raw;
-    else if constexpr (shifted(S)) return St::dec(q, raw, St::vel(src, p.N)[cell]);
-    else return St::dec(p, q, raw);
+    if constexpr (S == LBM_STORE_F16E8) {
+        float a, b, e[9];
+        e8_unpack(r.v, a, b);
+        e8_shifts(a, b, e);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) v[q] = add_lo(e[q], __builtin_bit_cast(uint16_t, r.q[q]));
+    } else {
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            if constexpr (S == LBM_STORE_F64 || S == LBM_STORE_F32) v[q] = r.q[q];
+            else if constexpr (S == LBM_STORE_F16) v[q] = from_half(__builtin_bit_cast(uint16_t, r.q[q]));
+            else if constexpr (shifted(S)) v[q] = St::dec(q, r.q[q], (typename Vel<S>::w_t)r.v);
+            else v[q] = St::dec(p, q, r.q[q]);
+        }
+    }
+}
+
+// w: pairs (1,2) (3,4) (5,6) (7,8), then 0
+template <class E>
+__device__ __forceinline__ void tile_store_halves(const Params &p, E *dst, int cell, const uint32_t *w)
+{
+    const uint32_t off = (uint32_t)opaque(cell) * 2u;
+    st_off(sbase(dst), off, (uint16_t)w[4]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        st_off(sbase(dst + (size_t)(2 * j + 1) * p.N), off, (uint16_t)w[j]);
+        st_off(sbase(dst + (size_t)(2 * j + 2) * p.N), off, (uint16_t)(w[j] >> 16));
+    }
 }
 
 // Post-collision values of one node: to LDS as the next iteration's pulls
@@ -59,9 +106,9 @@ __device__ __forceinline__ void tile_store(const Params &p, bool last, int cell,
     using St = Store<S>;
     using s_t = typename St::s_t;
     s_t *dst = static_cast<s_t *>(p.dst);
-    const uint32_t off = (uint32_t)cell * (uint32_t)sizeof(s_t);
     if constexpr (S == LBM_STORE_F32) {
         if (last) {
+            const uint32_t off = (uint32_t)opaque(cell) * 4u;
 #pragma unroll
             for (int q = 0; q < 9; ++q) st_off(sbase(dst + (size_t)q * p.N), off, h[q]);
         } else {
@@ -78,27 +125,52 @@ __device__ __forceinline__ void tile_store(const Params &p, bool last, int cell,
             v = Vel<S>::pack(ux, uy);
             Vel<S>::unpack(v, a, b);
         }
-        _Float16 raw[9];
         float e[9];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            if constexpr (S == LBM_STORE_F16E8) e[q] = e8_shift(q, a, b);
-            else e[q] = eq_shift(q, a, b);
-            raw[q] = to_half(h[q] - e[q]);
-        }
-        if (last) {
-            reinterpret_cast<w_t *>(dst + vel_offset(p.N))[cell] = v;
-#pragma unroll
-            for (int q = 0; q < 9; ++q) st_off(sbase(dst + (size_t)q * p.N), off, raw[q]);
+        if constexpr (S == LBM_STORE_F16E8) {
+            e8_shifts(a, b, e);
         } else {
 #pragma unroll
-            for (int q = 0; q < 9; ++q) lds[q * CAP + li] = e[q] + (float)raw[q];
+            for (int q = 0; q < 9; ++q) e[q] = eq_shift(q, a, b);
+        }
+        uint32_t w[5];                          // pairs (1,2) (3,4) (5,6) (7,8); 0
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            w[j] = to_half2(h[2 * j + 1] - e[2 * j + 1], h[2 * j + 2] - e[2 * j + 2]);
+        w[4] = __builtin_bit_cast(uint16_t, to_half(h[0] - e[0]));
+        if (last) {
+            st_off(sbase(dst + vel_offset(p.N)), (uint32_t)opaque(cell) * (uint32_t)sizeof(w_t), v);
+            tile_store_halves(p, dst, cell, w);
+        } else {
+            lds[li] = add_lo(e[0], w[4]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int q = 2 * j + 1;
+                lds[q * CAP + li] = add_lo(e[q], w[j]);
+                lds[(q + 1) * CAP + li] = add_hi(e[q + 1], w[j]);
+            }
+        }
+    } else if constexpr (S == LBM_STORE_F16) {
+        uint32_t w[5];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = to_half2(h[2 * j + 1], h[2 * j + 2]);
+        w[4] = __builtin_bit_cast(uint16_t, to_half(h[0]));
+        if (last) {
+            tile_store_halves(p, dst, cell, w);
+        } else {
+            const auto half = [](uint32_t u) { return (float)__builtin_bit_cast(_Float16, (uint16_t)u); };
+            lds[li] = half(w[4]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                lds[(2 * j + 1) * CAP + li] = half(w[j]);
+                lds[(2 * j + 2) * CAP + li] = half(w[j] >> 16);
+            }
         }
     } else {
         s_t raw[9];
 #pragma unroll
         for (int q = 0; q < 9; ++q) raw[q] = St::enc(p, q, h[q]);
         if (last) {
+            const uint32_t off = (uint32_t)opaque(cell) * (uint32_t)sizeof(s_t);
 #pragma unroll
             for (int q = 0; q < 9; ++q) st_off(sbase(dst + (size_t)q * p.N), off, raw[q]);
         } else {
@@ -118,9 +190,9 @@ __device__ __forceinline__ void tile_collide(const Params &p, bool last, int cel
         collide_f64(p, v, o, r, ux, uy);
         double *dst = static_cast<double *>(p.dst);
         if (last) {
+            const uint32_t off = (uint32_t)opaque(cell) * 8u;
 #pragma unroll
-            for (int q = 0; q < 9; ++q)
-                st_off(sbase(dst + (size_t)q * p.N), (uint32_t)cell * 8u, o[q]);
+            for (int q = 0; q < 9; ++q) st_off(sbase(dst + (size_t)q * p.N), off, o[q]);
         } else {
 #pragma unroll
             for (int q = 0; q < 9; ++q) lds[q * CAP + li] = o[q];
@@ -207,15 +279,6 @@ __device__ __forceinline__ int tile_last_level(const TileDesc &D, int K, int lev
     return lm;
 }
 
-// A copy the compiler knows nothing about: what is derived from it inside a
-// rarely taken branch of the iteration loop is not computed ahead of the loop
-// by every work-item (in registers every wave then pays for).
-__device__ __forceinline__ int opaque(int v)
-{
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
 // NT work-items, M nodes each, regions of up to CAP = NT * M nodes.
 template <int S, int NT, int M, bool LINKS>
 __device__ __forceinline__ void tile_run(const Params &p, const TileDesc &D,
@@ -238,7 +301,7 @@ __device__ __forceinline__ void tile_run(const Params &p, const TileDesc &D,
     const int base = *(const __attribute__((address_space(4))) int *)p.base;
 
     // ---- load r0: all planes of all nodes in flight
-    T v[M][9];
+    Raw<S> raw[M];
     {
         const uint32_t mg = D.mh[lev0];
 #pragma unroll
@@ -246,10 +309,7 @@ __device__ __forceinline__ void tile_run(const Params &p, const TileDesc &D,
             const int n = tid + m * NT;
             const int x = (int)__umulhi((uint32_t)n, mg), y = n - x * h0;
             const int cell = (r0.x + x) * ny + r0.y + y;
-            if (n < a0) {
-#pragma unroll
-                for (int q = 0; q < 9; ++q) v[m][q] = tile_load<S>(p, q, cell);
-            }
+            if (n < a0) tile_load<S>(p, cell, raw[m]);
         }
     }
     const TilePerim P = tile_perim(r1, nx, ny);
@@ -348,10 +408,12 @@ __device__ __forceinline__ void tile_run(const Params &p, const TileDesc &D,
     if (in_at >= 0) s_in[in_at] = T(in_v);
 #pragma unroll
     for (int m = 0; m < M; ++m) {
-        const int n = tid + m * NT;
+        const int n = opaque(tid + m * NT);      // (so that no decoding moves up to its loads)
         if (n < a0) {
+            T v[9];
+            tile_decode<S>(p, raw[m], v);
 #pragma unroll
-            for (int q = 0; q < 9; ++q) lds[q * CAP + n] = v[m][q];
+            for (int q = 0; q < 9; ++q) lds[q * CAP + n] = v[q];
         }
     }
     __syncthreads();
