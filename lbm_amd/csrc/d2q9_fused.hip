@@ -50,7 +50,7 @@ template <int S> __global__ __launch_bounds__(256) void k_init(Params p)
     T f[9];
 #pragma unroll
     for (int q = 0; q < 9; ++q)
-        f[q] = p.g0 ? T(p.g0[(size_t)q * p.N + cell]) : weight<T>(q);
+        f[q] = p.g0 ? T(__builtin_nontemporal_load(&p.g0[(size_t)q * p.N + cell])) : weight<T>(q);
     collide_any<S>(p, cell, f, p.rho_out != nullptr);
 }
 
@@ -78,12 +78,16 @@ __global__ __launch_bounds__(256) void k_batch_init(const Params *__restrict__ c
 // lattices (27 planes of doubles in FP64; 8192x2048: 4.2 TB/s); the inner
 // nodes, whose pulls need no bounds, issue all their loads together, and only
 // the perimeter waits for the ring row (FP64 8192x2048 1075 -> 864 us, a
-// cavity of the 256-case FP32 batch 19.8 -> 12.6).
+// cavity of the 256-case FP32 batch 19.8 -> 12.6).  Nobody reads the outputs
+// soon: they go past the caches.
 template <int S> __global__ __launch_bounds__(256) void k_epilogue(Params p)
 {
     using St = Store<S>;
     using T = typename St::T;
-    const int cell = blockIdx.x * 256 + threadIdx.x;
+    // contiguous slabs per XCD pay where the outputs are most of the traffic
+    // (batch 12.6 -> 11.0 us, F16 8192x2048 611 -> 573), in FP64 not (845, 921)
+    const int tile = S == LBM_STORE_F64 ? (int)blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
+    const int cell = tile * 256 + threadIdx.x;
     if (cell >= p.N) return;
     const int lx = p.nx - 1, ly = p.ny - 1;
     const auto *src = static_cast<const typename St::s_t *>(p.src);
@@ -121,8 +125,8 @@ template <int S> __global__ __launch_bounds__(256) void k_epilogue(Params p)
     }
 #pragma unroll
     for (int q = 0; q < 9; ++q) {
-        p.g_out[(size_t)q * p.N + cell] = (double)f[q];
-        p.gup_out[(size_t)q * p.N + cell] = up[q];
+        __builtin_nontemporal_store((double)f[q], &p.g_out[(size_t)q * p.N + cell]);
+        __builtin_nontemporal_store(up[q], &p.gup_out[(size_t)q * p.N + cell]);
     }
 }
 

@@ -780,8 +780,9 @@ __device__ __forceinline__ void collide_h(const Coll &k, float *h, float &rho, f
                                           float &uy)
 {
     const float drho = ((h[0] + h[1]) + (h[2] + h[3])) + ((h[4] + h[5]) + (h[6] + h[7])) + h[8];
-    const float jx = (h[1] - h[2]) + (h[5] - h[6]) + (h[8] - h[7]);
-    const float jy = (h[3] - h[4]) + (h[5] - h[6]) + (h[7] - h[8]);
+    const float d78 = h[7] - h[8];
+    const float jx = (h[1] - h[2]) + (h[5] - h[6]) - d78;
+    const float jy = (h[3] - h[4]) + (h[5] - h[6]) + d78;
     rho = 1.0f + drho;
     const float inv = __builtin_amdgcn_rcpf(rho);
     ux = jx * inv;
