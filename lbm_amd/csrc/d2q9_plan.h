@@ -273,7 +273,9 @@ struct TileKind {
 //   FP64  100^2 K7 512x1 1.64 (7.0), 5 iterations 1.80, 3 1.98;
 //         151^2 K7 512x2 1.81, K5 512x1 1.87 (6.9);
 //         200^2 K5 512x2 2.03, K7 512x2 2.18, K3 512x1 2.35 (7.0);
-//         400^2 K5 1024x2 3.47, K5 512x2 3.92 (9.0);
+//         300^2 K5 512x2 2.66, K7 1024x2 2.69; 400^2 K7 1024x2 3.35, K5 3.35,
+//         K5 512x2 3.92 (9.0); 1073x200 (links) K7 1024x2 4.09, K5 4.67;
+//         600^2 K3 1024x2 6.45, K3 512x2 8.27; 800^2 K3 512x2 10.3, 1024x2 11.6;
 //         8192x2048 K3 512x2 237, K5 512x2 248, K5 1024x2 284, K3 512x1 307 (434)
 //   FP32  100^2 K7 512x1 1.26 (9.0); 200^2 K7 1024x2 1.45, 512x2 1.56 (8.9);
 //         1073x240 (links) K5 1024x2 3.30, K7 1024x4 3.59; 700^2 K7 1024x4 4.03 (12.7);
@@ -284,7 +286,9 @@ inline const TileKind *tile_kinds(bool f64, int &n)
     static const TileKind d[] = {{0, 7, 512, 512, 512, 0},
                                  {1, 7, 1024, 512, 600, 0},
                                  {1, 5, 1024, 512, 1024, 0},
+                                 {2, 7, 2048, 1024, 2048, 0},
                                  {2, 5, 2048, 1024, 2048, 0},
+                                 {2, 3, 2048, 1024, 2048, 0},
                                  {1, 3, 1024, 512, 1024, 1}};
     static const TileKind f[] = {{0, 7, 512, 512, 512, 0},
                                  {1, 7, 1024, 512, 640, 0},
@@ -292,7 +296,7 @@ inline const TileKind *tile_kinds(bool f64, int &n)
                                  {2, 5, 2048, 1024, 2048, 0},
                                  {4, 7, 4096, 1024, 4096, 0},
                                  {3, 5, 2048, 512, 2048, 1}};
-    n = f64 ? 5 : 6;
+    n = f64 ? 7 : 6;
     return f64 ? d : f;
 }
 

@@ -110,6 +110,14 @@ def test_several_tiles_per_cu(storage):
     _same(_run(nx, ny, storage, 9, squares)[0], _run(nx, ny, storage, 9, squares, single=True)[0], storage)
 
 
+@pytest.mark.parametrize("storage,nx,ny", [("f64", 530, 519), ("f32", 530, 519), ("f64", 601, 600)])
+def test_largest_single_round(storage, nx, ny):
+    """Lattices whose largest regions just fit a work-group: fewer iterations."""
+    squares = ((3, 300, 30), (250, 200, 60), (480, 470, 40))
+    _same(_run(nx, ny, storage, 11, squares)[0], _run(nx, ny, storage, 11, squares, single=True)[0],
+          (nx, ny, storage))
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 15])
 def test_every_remainder(n):
     kw = dict(squares=((10, 12, 6),), pressure=False, pool=True)
