@@ -133,16 +133,20 @@ LBM_HD inline bool tile_perim_node(const TileRect &r, const TilePerim &P, int n,
     return true;
 }
 
+// A link near a tile: its node and the far end of its stencil.
+struct NearLink {
+    int x, y, fx, fy;
+    const PlanLink *link;
+};
+
 // Plans the tile of nodes [xa, xb) x [ya, yb): adds it to the plan, or its two
 // halves where a link stencil makes it larger than the shape allows.
 // recip[h] = 2^32 / h.  near: the links (sorted as the lattice's) within 2 K + 2 nodes of the tile,
 // at least: a level's stencils reach two nodes beyond the next one.
-inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<const PlanLink *> &near,
+inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<NearLink> &near,
                      const std::vector<uint32_t> &recip, int cse, int xa, int xb, int ya, int yb,
                      TilePlan &out)
 {
-    static const int cx[9] = {0, 1, -1, 0, 0, 1, -1, -1, 1};
-    static const int cy[9] = {0, 0, 0, 1, -1, 1, -1, 1, -1};
     static const int ns[9] = {0, 2, 1, 4, 3, 6, 5, 8, 7};
     if (xb - xa < 2 || yb - ya < 2) return false;
     out.tiles.emplace_back();
@@ -159,16 +163,12 @@ inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<const
         int px = std::max(lo_x - 1, 0), qx = std::min(hi_x + 1, nx - 1);
         int py = std::max(lo_y - 1, 0), qy = std::min(hi_y + 1, ny - 1);
         const int px0 = px, qx0 = qx, py0 = py, qy0 = qy;
-        for (const PlanLink *n : near) {
-            const PlanLink &L = *n;
-            if (L.x < lo_x || L.x > hi_x || L.y < lo_y || L.y > hi_y || !L.mode) continue;
-            const int far = L.mode == 1 ? 2 : 1, qb = ns[L.q];
-            const int fx = L.x + far * cx[qb], fy = L.y + far * cy[qb];
-            if (fx < 0 || fx >= nx || fy < 0 || fy >= ny) return false;
-            px = std::min(px, fx);
-            qx = std::max(qx, fx);
-            py = std::min(py, fy);
-            qy = std::max(qy, fy);
+        for (const NearLink &L : near) {
+            if (L.x < lo_x || L.x > hi_x || L.y < lo_y || L.y > hi_y) continue;
+            px = std::min(px, L.fx);
+            qx = std::max(qx, L.fx);
+            py = std::min(py, L.fy);
+            qy = std::max(qy, L.fy);
         }
         // a wall node beside a corner carries the corner's adjoint
         if (s.adjoint && (py == 0 || qy == ny - 1)) {
@@ -189,10 +189,10 @@ inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<const
     const TileRect &r0 = d.r[0], &r1 = d.r[1];
     const TilePerim P = tile_perim(s.adjoint ? r0 : r1, nx, ny);
     bool fits = (int64_t)r0.w * r0.h <= s.cap && P.slots <= s.nt && P.slots + P.inner <= s.cap;
-    const auto inside = [&](const PlanLink &L) {
+    const auto inside = [&](const NearLink &L) {
         return L.x >= r1.x && L.x < r1.x + r1.w && L.y >= r1.y && L.y < r1.y + r1.h;
     };
-    for (const PlanLink *n : near) d.n_links += inside(*n);
+    for (const NearLink &n : near) d.n_links += inside(n);
     fits = fits && d.n_links <= s.nt;
     if (!fits) {
         out.tiles.pop_back();
@@ -213,9 +213,9 @@ inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<const
     if (d.n_links) {
         out.nodes.resize(out.nodes.size() + (size_t)r0.w * r0.h, 0u);
         int n = 0;
-        for (const PlanLink *l : near) {
-            const PlanLink &L = *l;
-            if (!inside(L)) continue;
+        for (const NearLink &l : near) {
+            if (!inside(l)) continue;
+            const PlanLink &L = *l.link;
             const bool own = L.x >= xa && L.x < xb && L.y >= ya && L.y < yb;
             TileLink t{};
             t.x = (int16_t)(L.x - r0.x);
@@ -343,41 +343,35 @@ inline bool plan_tiles(int nx, int ny, const TileShape &s, const std::vector<Pla
         v = std::min(std::max(v, 0), n - 1);
         return (int)((((int64_t)v + 1) * nt - 1) / n);
     };
-    // the links of each tile: order[first[t] .. first[t + 1])
-    std::vector<int> first((size_t)s.ntx * s.nty + 1, 0), order(links.size());
-    const auto tile = [&](const PlanLink &L) {
-        return (size_t)tile_of(L.x, nx, s.ntx) * s.nty + tile_of(L.y, ny, s.nty);
-    };
-    for (const PlanLink &L : links) ++first[tile(L) + 1];
-    for (size_t t = 1; t < first.size(); ++t) first[t] += first[t - 1];
-    std::vector<int> at(first);
-    for (size_t k = 0; k < links.size(); ++k) order[at[tile(links[k])]++] = (int)k;
+    static const int cx[9] = {0, 1, -1, 0, 0, 1, -1, -1, 1};
+    static const int cy[9] = {0, 0, 0, 1, -1, 1, -1, 1, -1};
+    static const int ns[9] = {0, 2, 1, 4, 3, 6, 5, 8, 7};
+    std::vector<NearLink> all;
+    all.reserve(links.size());
+    for (const PlanLink &L : links) {
+        const int far = L.mode == 1 ? 2 : L.mode ? 1 : 0, qb = ns[L.q];
+        const NearLink n{L.x, L.y, L.x + far * cx[qb], L.y + far * cy[qb], &L};
+        if (n.fx < 0 || n.fx >= nx || n.fy < 0 || n.fy >= ny) return false;
+        all.push_back(n);
+    }
+    const size_t need = out.tiles.size() + (size_t)s.ntx * s.nty;
+    if (need > out.tiles.capacity()) out.tiles.reserve(std::max(need, 2 * out.tiles.capacity()));
     const int margin = 2 * s.K + 2;
-    std::vector<const PlanLink *> near;
-    std::vector<int> ks;
+    std::vector<std::vector<NearLink>> near(s.nty);  // of a column's tiles, in the links' order
     std::vector<uint32_t> recip(ny + 1, 0u);         // 2^32 / height
     for (int h = 1; h <= ny; ++h) recip[h] = 0xffffffffu / (uint32_t)h + 1u;
+    const auto before = [](const NearLink &L, int x) { return L.x < x; };
     for (int tx = 0; tx < s.ntx; ++tx) {
         const int xa = (int)((int64_t)nx * tx / s.ntx), xb = (int)((int64_t)nx * (tx + 1) / s.ntx);
-        const int ta = tile_of(xa - margin, nx, s.ntx), tb = tile_of(xb + margin, nx, s.ntx);
+        for (auto &n : near) n.clear();
+        for (auto l = std::lower_bound(all.begin(), all.end(), xa - margin, before);
+             l != all.end() && l->x < xb + margin; ++l)
+            for (int ty = tile_of(l->y - margin, ny, s.nty); ty <= tile_of(l->y + margin, ny, s.nty); ++ty)
+                near[ty].push_back(*l);
         for (int ty = 0; ty < s.nty; ++ty) {
             const int ya = (int)((int64_t)ny * ty / s.nty),
                       yb = (int)((int64_t)ny * (ty + 1) / s.nty);
-            const int ua = tile_of(ya - margin, ny, s.nty), ub = tile_of(yb + margin, ny, s.nty);
-            ks.clear();
-            for (int t = ta; t <= tb; ++t) {
-                const size_t lo = (size_t)t * s.nty + ua, hi = (size_t)t * s.nty + ub;
-                for (int i = first[lo]; i < first[hi + 1]; ++i) {
-                    const PlanLink &L = links[order[i]];
-                    if (L.x >= xa - margin && L.x < xb + margin && L.y >= ya - margin &&
-                        L.y < yb + margin)
-                        ks.push_back(order[i]);
-                }
-            }
-            std::sort(ks.begin(), ks.end());
-            near.clear();
-            for (int k : ks) near.push_back(&links[k]);
-            if (!plan_one(nx, ny, s, near, recip, cse, xa, xb, ya, yb, out)) return false;
+            if (!plan_one(nx, ny, s, near[ty], recip, cse, xa, xb, ya, yb, out)) return false;
         }
     }
     return true;
