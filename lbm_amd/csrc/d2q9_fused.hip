@@ -1248,9 +1248,18 @@ int build_tiles(const std::vector<lbm_fused *> &cases, TileSet &t, int64_t *byte
     LBM_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     LBM_HIP_TRY(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     std::vector<PlanCase> pc;
+    int64_t total = 0;
     for (lbm_fused *h : cases) {
         pc.push_back(PlanCase{h->nx, h->ny, &h->plan_links});
         t.links = t.links || h->n_links > 0;
+        total += h->N;
+    }
+    // Q16's coding costs more arithmetic than the bytes it saves once the
+    // lattice takes many rounds (us per iteration, one per launch first:
+    // 2000x1000 19.4, 17.5; 2600x1100 22.0, 23.9; 8192x2048 111, 130)
+    if (cases[0]->storage == LBM_STORE_Q16 && total > 2000000) {
+        for (lbm_fused *h : cases) std::vector<PlanLink>().swap(h->plan_links);
+        return LBM_OK;
     }
     const bool f64 = cases[0]->storage == LBM_STORE_F64;
     TilePlan plan;

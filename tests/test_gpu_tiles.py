@@ -118,6 +118,12 @@ def test_largest_single_round(storage, nx, ny):
           (nx, ny, storage))
 
 
+@pytest.mark.parametrize("nx,ny", [(1999, 1000), (2003, 1000)])
+def test_q16_either_side_of_one_iteration_launches(nx, ny):
+    squares = ((3, 300, 30), (900, 200, 90), (1900, 900, 40))
+    _same(_run(nx, ny, "q16", 9, squares)[0], _run(nx, ny, "q16", 9, squares, single=True)[0], nx)
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 15])
 def test_every_remainder(n):
     kw = dict(squares=((10, 12, 6),), pressure=False, pool=True)
