@@ -13,7 +13,8 @@ precision f - w - E(v) with the node velocity v in a half pair), f16e8 (the
 same with v as an 8-bit pair) and Q16 (16-bit fixed point of f - w) forms are
 timed on the same workload and reported under "forms", each with its
 fraction of the 8 TB/s HBM roofline (algorithmic bytes per lattice update:
-18 x storage bytes, 44 for f16e, 40 for f16e8), its drag error against the
+18 x storage bytes, 44 for f16e, 40 for f16e8; a launch of several iterations
+moves them once, so this rate can pass the peak), its drag error against the
 FP64 run and its velocity-field L2 error.  Further sections: the 200x200
 cavity, the Turek cylinder through the drop-in lattice/run, the Turek
 cylinder per form (shedding statistics), a 256-cavity batch and the adjoint;
@@ -583,8 +584,13 @@ def summarize_profile(pdir, nodes, copy_bytes=2 << 30):
         return out
 
     def form_of(name):
+        # form, nodes per work-item, iterations per launch (this array's shapes)
+        m = re.search(r"k_tile<(\d), \d+, (\d), \w+>", name)
+        if m:
+            form = FORM_OF_STORE[m.group(1)]
+            return form, m.group(2), 3 if form == "f64" else 5
         m = re.search(r"k_step(_v4|_w7|_w8)?<(\d), (\d)>", name)
-        return (FORM_OF_STORE[m.group(2)], m.group(1) == "_v4", int(m.group(3))) if m else None
+        return (FORM_OF_STORE[m.group(2)], m.group(3) + (m.group(1) or ""), 1) if m else None
 
     stats = {r["Name"]: r for r in rows("trace", "kernel_stats.csv")}
     counters = {}
@@ -606,16 +612,17 @@ def summarize_profile(pdir, nodes, copy_bytes=2 << 30):
              f"Counter calibration on the copy kernel (k_copy16, {copy_bytes >> 20} MiB read and "
              f"{copy_bytes >> 20} MiB written per dispatch): FETCH_SIZE x {fetch_factor:.3f}, "
              f"WRITE_SIZE x {write_factor:.3f}.", "",
-             "| kernel | form | calls | avg us | min us | max us | algorithmic MB/launch "
-             "| HBM read MB | HBM write MB | traffic / algorithmic | algorithmic GB/s |",
-             "|---|---|---|---|---|---|---|---|---|---|---|"]
+             "| kernel | form | iterations/launch | calls | avg us | min us | max us "
+             "| algorithmic MB/launch | HBM read MB | HBM write MB | traffic / algorithmic "
+             "| algorithmic GB/s |",
+             "|---|---|---|---|---|---|---|---|---|---|---|---|"]
     traffic = {}
-    for name, st in sorted(stats.items()):
+    for name, st in sorted(stats.items(), key=lambda e: (form_of(e[0]) or ("", "", 0))[2]):
         fm = form_of(name)
         if fm is None:
             continue
-        form, v4, cpt = fm
-        alg = float(BYTES_PER_UPDATE[form]) * nodes
+        form, cpt, its = fm
+        alg = float(BYTES_PER_UPDATE[form]) * nodes * its
         avg_us = float(st["AverageNs"]) / 1e3
         fb = counters["FETCH_SIZE"].get(name)
         wb = counters["WRITE_SIZE"].get(name)
@@ -623,12 +630,13 @@ def summarize_profile(pdir, nodes, copy_bytes=2 << 30):
         wr = wb * 1024.0 * write_factor if wb is not None else None
         tot = rd + wr if rd is not None and wr is not None else None
         lines.append(
-            f"| `{name}` | {form}{' 4-node' if v4 else ''} cpt {cpt} | {st['Calls']} | "
+            f"| `{name}` | {form} cpt {cpt} | {its} | {st['Calls']} | "
             f"{avg_us:.2f} | {float(st['MinNs']) / 1e3:.2f} | {float(st['MaxNs']) / 1e3:.2f} | "
             f"{alg / 1e6:.1f} | {rd / 1e6 if rd else float('nan'):.1f} | "
             f"{wr / 1e6 if wr else float('nan'):.1f} | "
             f"{tot / alg if tot else float('nan'):.3f} | {alg / (avg_us * 1e-6) / 1e9:.1f} |")
-        traffic[form] = {"kernel": name, "avg_duration_us": round(avg_us, 3),
+        traffic[form] = {"kernel": name, "iterations_per_launch": its,
+                         "avg_duration_us": round(avg_us, 3),
                          "algorithmic_bytes_per_launch": alg,
                          "hbm_read_bytes_per_launch": rd, "hbm_write_bytes_per_launch": wr,
                          "hbm_bytes_per_launch": tot}
@@ -750,7 +758,10 @@ def main():
     tpath = os.path.join(ROOT, "profiles", "fused_f16_obstacle_array_traffic.json")
     if os.path.exists(tpath):
         with open(tpath) as fh:
-            traffic = json.load(fh).get("hbm_bytes_per_launch")
+            t = json.load(fh)
+            traffic = t.get("hbm_bytes_per_launch")
+            if traffic:
+                traffic /= t.get("iterations_per_launch", 1)       # of one iteration
     cpu = None
     if not args.no_cpu:
         print(f"# cpu baseline: oracle, {args.cpu_iterations} iterations", file=sys.stderr,

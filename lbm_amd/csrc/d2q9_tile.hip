@@ -16,10 +16,11 @@
 // rectangles, and pay the chain once; an iteration is then bound by the
 // collision's arithmetic, ~175 FP64 instructions per node, with 1.2-1.5 times
 // as many nodes computed as owned.  Measured per iteration (MI355X, one
-// iteration per launch in brackets): FP64 cavity 100x100 1.64 us (7.0),
-// 200x200 2.03 (7.0), Turek channel 1073x200 4.8 (10.7), 8192x2048 obstacle
-// array 237 (434); FP32 channel 541x101 1.9 (9.4), array 101 (211); FP16 array
-// 97-104 (110), f16e8 129 (148).
+// iteration per launch in brackets): FP64 cavity 100x100 1.7 us (7.0),
+// 200x200 1.9 (7.5), Turek channel 1073x200 4.1 (10.7), 8192x2048 obstacle
+// array 214 (428); FP32 channel 541x101 1.9 (9.4), array 83 (212); FP16 array
+// 88 (107), BF16 88 (112), f16e 116 (144), f16e8 115 (140).  On the array the
+// vector units are 60 (FP64) to 80 % (FP16) busy at the 1.9-2.2 GHz held.
 //
 // Layout: the nine planes of the rectangle lie one after the other in LDS, in
 // float or double.  Every work-item keeps its M nodes for the whole launch:
