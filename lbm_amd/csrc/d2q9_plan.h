@@ -133,9 +133,10 @@ LBM_HD inline bool tile_perim_node(const TileRect &r, const TilePerim &P, int n,
     return true;
 }
 
-// A link near a tile: its node and the far end of its stencil.
+// A link near a tile: its node, its stencil's direction and reach (0, 1, 2 nodes).
 struct NearLink {
-    int x, y, fx, fy;
+    int x, y;
+    int8_t dx, dy, reach;
     const PlanLink *link;
 };
 
@@ -154,22 +155,39 @@ inline bool plan_one(int nx, int ny, const TileShape &s, const std::vector<NearL
     d.cse = cse;
     d.regular = 1;
     int lo_x = xa, hi_x = xb - 1, lo_y = ya, hi_y = yb - 1;   // inclusive
+    static thread_local std::vector<int> far;
+    far.resize(4 * near.size());
+    int *const fx = far.data(), *const fy = fx + near.size(), *const dx = fy + near.size(),
+              *const dy = dx + near.size();
+    size_t n_far = 0;
+    for (const NearLink &L : near) {
+        if (L.reach != 2) continue;
+        fx[n_far] = L.x;
+        fy[n_far] = L.y;
+        dx[n_far] = L.dx;
+        dy[n_far++] = L.dy;
+    }
     for (int l = s.K; l >= 0; --l) {
         d.r[l] = TileRect{lo_x, lo_y, hi_x - lo_x + 1, hi_y - lo_y + 1};
         const int h = d.r[l].h, hi = h - (lo_y == 0) - (hi_y == ny - 1);
         d.mh[l] = recip[h];
         d.mi[l] = hi > 1 ? recip[hi] : 0u;
         if (l == 0) break;
-        int px = std::max(lo_x - 1, 0), qx = std::min(hi_x + 1, nx - 1);
-        int py = std::max(lo_y - 1, 0), qy = std::min(hi_y + 1, ny - 1);
-        const int px0 = px, qx0 = qx, py0 = py, qy0 = qy;
-        for (const NearLink &L : near) {
-            if (L.x < lo_x || L.x > hi_x || L.y < lo_y || L.y > hi_y) continue;
-            px = std::min(px, L.fx);
-            qx = std::max(qx, L.fx);
-            py = std::min(py, L.fy);
-            qy = std::max(qy, L.fy);
+        // a stencil of two nodes reaches beyond the next level from the edge only
+        int wide = 0;
+        for (size_t i = 0; i < n_far; ++i) {
+            const int x = fx[i], y = fy[i];
+            const int in = (x >= lo_x) & (x <= hi_x) & (y >= lo_y) & (y <= hi_y);
+            const int w = ((x == lo_x) & (dx[i] < 0)) | ((x == hi_x) & (dx[i] > 0)) << 1 |
+                          ((y == lo_y) & (dy[i] < 0)) << 2 | ((y == hi_y) & (dy[i] > 0)) << 3;
+            wide |= -in & w;
         }
+        int px = wide & 1 ? lo_x - 2 : std::max(lo_x - 1, 0);
+        int qx = wide & 2 ? hi_x + 2 : std::min(hi_x + 1, nx - 1);
+        int py = wide & 4 ? lo_y - 2 : std::max(lo_y - 1, 0);
+        int qy = wide & 8 ? hi_y + 2 : std::min(hi_y + 1, ny - 1);
+        if (wide) d.regular = 0;
+        const int px0 = px, qx0 = qx, py0 = py, qy0 = qy;
         // a wall node beside a corner carries the corner's adjoint
         if (s.adjoint && (py == 0 || qy == ny - 1)) {
             if (px == 1) px = 0;
@@ -350,12 +368,19 @@ inline bool plan_tiles(int nx, int ny, const TileShape &s, const std::vector<Pla
     all.reserve(links.size());
     for (const PlanLink &L : links) {
         const int far = L.mode == 1 ? 2 : L.mode ? 1 : 0, qb = ns[L.q];
-        const NearLink n{L.x, L.y, L.x + far * cx[qb], L.y + far * cy[qb], &L};
-        if (n.fx < 0 || n.fx >= nx || n.fy < 0 || n.fy >= ny) return false;
+        const int x = L.x + far * cx[qb], y = L.y + far * cy[qb];
+        if (x < 0 || x >= nx || y < 0 || y >= ny) return false;
+        const NearLink n{L.x, L.y, (int8_t)cx[qb], (int8_t)cy[qb], (int8_t)far, &L};
         all.push_back(n);
     }
-    const size_t need = out.tiles.size() + (size_t)s.ntx * s.nty;
-    if (need > out.tiles.capacity()) out.tiles.reserve(std::max(need, 2 * out.tiles.capacity()));
+    // room at once (fresh pages cost more than what is written to them): a link
+    // lies in about two tiles' regions, which hold some 20 nodes per link
+    const auto room = [](auto &v, size_t n) {
+        if (v.size() + n > v.capacity()) v.reserve(std::max(v.size() + n, 2 * v.capacity()));
+    };
+    room(out.tiles, (size_t)s.ntx * s.nty);
+    room(out.links, 2 * links.size());
+    room(out.nodes, 20 * links.size());
     const int margin = 2 * s.K + 2;
     std::vector<std::vector<NearLink>> near(s.nty);  // of a column's tiles, in the links' order
     std::vector<uint32_t> recip(ny + 1, 0u);         // 2^32 / height
